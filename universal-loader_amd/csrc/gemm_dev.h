@@ -9,6 +9,25 @@
 #include "ulspec_internal.h"
 
 namespace ulspec {
+
+// Arguments of the dequant-GEMM kernels (see the X operand below).
+struct GemmArgs {
+    const uint8_t* w;
+    uint32_t w_bytes;
+    const _Float16* x;
+    float* out;  // Y, or the slice partials [ks_count][M][N] of the split-K kernel
+    int M, N, K, n_tiles, n_chunks, ks_count;
+    int ks_q, ks_r;  // n_chunks = ks_q * ks_count + ks_r; slice s starts at s * ks_q + min(s, ks_r)
+    int hl;          // split X (see above)
+    int lo_rows;     // split X: row of X holding the low part of row 0
+    int xrows;       // rows of X staged: M, or 2M when split
+    GemmFuse f;      // row scale and epilogue
+};
+
+// The sum of a.ks_count slices of part [ks][M][N] (host; asynchronous), row
+// scale and a.f's epilogue into a.out.
+void gemm_reduce_launch(ulspec_ctx* ctx, const GemmArgs& a, const float* part);
+
 namespace {
 
 constexpr int kQ40Chunk = 1152;
@@ -185,19 +204,6 @@ __device__ __forceinline__ half8_t dequant_q4_k(uint32_t v, const SubScale& s, c
 // rows, and the two halves of the result are added in the epilogue (hi + lo *
 // 2^-11), so M <= 8 per 16-column tile.
 constexpr uint32_t kOOB = 0x80000000u;  // >= any buffer's num_records
-
-struct GemmArgs {
-    const uint8_t* w;
-    uint32_t w_bytes;
-    const _Float16* x;
-    float* out;  // Y, or the slice partials [ks_count][M][N] of the split-K kernel
-    int M, N, K, n_tiles, n_chunks, ks_count;
-    int ks_q, ks_r;  // n_chunks = ks_q * ks_count + ks_r; slice s starts at s * ks_q + min(s, ks_r)
-    int hl;          // split X (see above)
-    int lo_rows;     // split X: row of X holding the low part of row 0
-    int xrows;       // rows of X staged: M, or 2M when split
-    GemmFuse f;      // row scale and epilogue
-};
 
 // X row behind staged row rho (0 .. xrows-1).
 __device__ __forceinline__ int x_row(const GemmArgs& a, int rho)

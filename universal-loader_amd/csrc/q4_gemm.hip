@@ -1464,7 +1464,7 @@ ulspec_status gemm_init(ulspec_ctx* ctx)
                                     (int)(kWideLdsMax - at.sharedSizeBytes));
             if (e != hipSuccess) return hip_fail(ctx, e, "hipFuncSetAttribute(max dynamic LDS)");
         }
-    return ULSPEC_OK;
+    return gemm_tile_init(ctx);
 }
 
 // Launch a whole-X kernel if one fits; false when the split-K path must run.
@@ -1611,6 +1611,23 @@ void reduce_launch(const GemmArgs& a, const float* part, int cols, bool four_row
         hipLaunchKernelGGL((gemm_reduce_kernel<KB, 1>), dim3(cols, a.M), dim3(256), 0, st, a, part);
 }
 
+}  // namespace
+
+// The sum of a.ks_count slices of part [ks][M][N], row scale and a.f's
+// epilogue into a.out.
+void gemm_reduce_launch(ulspec_ctx* ctx, const GemmArgs& a, const float* part)
+{
+    const int cols = (16 * a.n_tiles + 255) / 256;
+    const bool wide = cols * ((a.M + 3) / 4) >= 2 * std::max(1, ctx->n_cu);
+    if (a.ks_count <= 2) reduce_launch<2>(a, part, cols, wide, ctx->stream);
+    else if (a.ks_count <= 4) reduce_launch<4>(a, part, cols, wide, ctx->stream);
+    else if (a.ks_count <= 8) reduce_launch<8>(a, part, cols, wide, ctx->stream);
+    else if (a.ks_count <= 16) reduce_launch<16>(a, part, cols, wide, ctx->stream);
+    else reduce_launch<kMaxSlices>(a, part, cols, wide, ctx->stream);
+}
+
+namespace {
+
 // The split-K kernel over a.M rows into part[ks][M][N], then the slice sum, row
 // scale and a.f's epilogue into y (one slice, no row scale and a plain store:
 // straight into y).
@@ -1629,13 +1646,7 @@ void split_launch(ulspec_ctx* ctx, const Weight& w, GemmArgs a, float* part, flo
     else slice_launch_t<ULSPEC_GGML_F16>(a, mt, ctx->stream);
     if (direct) return;
     a.out = y;
-    const int cols = (16 * a.n_tiles + 255) / 256;
-    const bool wide = cols * ((a.M + 3) / 4) >= 2 * std::max(1, ctx->n_cu);
-    if (a.ks_count <= 2) reduce_launch<2>(a, part, cols, wide, ctx->stream);
-    else if (a.ks_count <= 4) reduce_launch<4>(a, part, cols, wide, ctx->stream);
-    else if (a.ks_count <= 8) reduce_launch<8>(a, part, cols, wide, ctx->stream);
-    else if (a.ks_count <= 16) reduce_launch<16>(a, part, cols, wide, ctx->stream);
-    else reduce_launch<kMaxSlices>(a, part, cols, wide, ctx->stream);
+    gemm_reduce_launch(ctx, a, part);
 }
 
 }  // namespace
@@ -1647,6 +1658,15 @@ ulspec_status gemm_launch(ulspec_ctx* ctx, const Weight& w, const uint16_t* x, u
     const _Float16* X = reinterpret_cast<const _Float16*>(x);
     if (gemm_workspace_bytes(w) > ctx->ws_bytes)
         return fail(ctx, ULSPEC_EINVAL, "verify_gemm: workspace smaller than the weight needs");
+    if (gemm_tile_wins(w, M)) {
+        const uint32_t step = std::min<uint32_t>(kTileRowsH16, (kOOB - 1) / (std::max(2 * w.k, 4 * w.n)));
+        for (uint32_t m0 = 0; m0 < M; m0 += step) {
+            const ulspec_status s = gemm_tile(ctx, w, GemmFuse(), x + (size_t)m0 * w.k, std::min(step, M - m0), false, 0,
+                                              y + (size_t)m0 * w.n, ctx->ws, ctx->ws_bytes);
+            if (s != ULSPEC_OK) return s;
+        }
+        return check_launch(ctx, "verify_gemm launch");
+    }
     for (uint32_t m0 = 0; m0 < M; m0 += kGemmRowsH16) {
         const uint32_t mc = std::min<uint32_t>(kGemmRowsH16, M - m0);
         GemmArgs a = make_args(w, X + (size_t)m0 * w.k, mc, false, 0, y + (size_t)m0 * w.n);
@@ -1737,7 +1757,8 @@ ulspec_status weight_create(ulspec_ctx* ctx, uint32_t type, const void* blocks, 
     // workspace: the host blocks (when not on the device), then for the fp16
     // formats the fp16 rows
     const size_t raw_room = on_device ? 0 : (nbytes + 255) / 256 * 256;
-    const size_t need = f16 ? raw_room + (size_t)N * K * 2 : std::max(raw_room, gemm_workspace_bytes(w));
+    const size_t need = std::max(f16 ? raw_room + (size_t)N * K * 2 : std::max(raw_room, gemm_workspace_bytes(w)),
+                                 gemm_tile_workspace_bytes(w, ctx->n_cu));
     ulspec_status st = workspace(ctx, need, &raw);
     if (st != ULSPEC_OK) {
         (void)hipFree(w.dev);

@@ -135,6 +135,15 @@ ulspec_status rows_to_f16(ulspec_ctx* ctx, uint32_t type, const void* raw, uint3
 // epilogue.
 ulspec_status gemm_fused(ulspec_ctx* ctx, const Weight& w, const GemmFuse& f, const uint16_t* x, uint32_t M,
                          uint32_t lo_rows, float* y);
+// The many-row dequant-GEMM (gemm_tile.hip): fp16 X (hl false) or split X (the
+// low part of row m at row lo_rows + m), at most kTileRowsH16 rows of fp16 X;
+// ws holds the row sums and, when K is split, the slice partials.
+constexpr uint32_t kTileRowsH16 = 4096;
+bool gemm_tile_wins(const Weight& w, uint32_t M);
+ulspec_status gemm_tile_init(ulspec_ctx* ctx);
+size_t gemm_tile_workspace_bytes(const Weight& w, int n_cu);
+ulspec_status gemm_tile(ulspec_ctx* ctx, const Weight& w, const GemmFuse& f, const uint16_t* x, uint32_t M, bool hl,
+                        uint32_t lo_rows, float* y, void* ws, size_t ws_bytes);
 size_t gemm_workspace_bytes(const Weight& w);
 uint32_t choose_ksplit(uint32_t n_tiles, uint32_t n_chunks, int n_cu);
 size_t gemm_split_part_bytes(const Weight& w, uint32_t M);
