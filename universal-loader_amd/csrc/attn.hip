@@ -30,6 +30,7 @@
 #include "hip_common.h"
 #include "ulspec_internal.h"
 
+#include <algorithm>
 #include <cmath>
 
 using namespace ulspec;
@@ -56,6 +57,7 @@ struct AttnArgs {
     int n_prefix, nq, L, H, Hkv, splits, keys_per_split;
     float scale_log2;   // scale * log2(e)
     int out_mode;
+    int q_tile;         // queries of one plan (kPromptQ of a prompt; 0: all of them)
     uint32_t mask[kMaxQ];
 };
 
@@ -272,6 +274,7 @@ __global__ __launch_bounds__(D) void attn_merge_kernel(AttnArgs a)
     const float mv = q0[ds * stride + D], lv = q0[ds * stride + D + 1];
     int n_prefix, L;
     attn_len(a, b, n_prefix, L);
+    if (a.q_tile) L = n_prefix + min(a.nq, qi / a.q_tile * a.q_tile + a.q_tile);  // the keys of its query tile
     const int ns = min(S, (L + a.keys_per_split - 1) / a.keys_per_split);
     if (d < S) {
         sm[d] = mv;
@@ -299,6 +302,199 @@ __global__ __launch_bounds__(D) void attn_merge_kernel(AttnArgs a)
     store_out<D>(a, (((size_t)b * a.nq + qi) * a.H + h) * D + d, o / Ls);
 }
 
+// Attention of a prompt's rows (nq of them behind n_prefix cached keys, causal).
+//
+// Grid (heads, query tiles, splits); a workgroup of 4 waves takes 128 queries
+// of one head, 32 per wave, over a key range in stages of 64 keys.  K and V of
+// the next stage go to the other LDS buffer by direct buffer->LDS copies while
+// a stage is multiplied (one barrier per stage):
+//   S^T[key][query] = K . Q^T         32x32x16 fp16 MFMA, Q^T in registers
+//   online softmax per query in the log2 domain (fp32); O is rescaled only in
+//   the stages where some query's maximum moved
+//   O^T[d][query] += V^T . P^T        the S^T accumulators are the P^T operand
+//                                     (its K slots are the keys 16 t + 8 (e / 4)
+//                                     + 4 kg + e % 4 of lane half kg), V^T by
+//                                     transposing LDS reads; P = P_hi + P_lo
+// LDS rows of D halfs in 16-byte units, unit u of K row r at u ^ (r & 15) (D =
+// 128) or u ^ ((r / 2) & 7) (D = 64): the 16 rows of an operand read take 16
+// bank groups; of V row r at u ^ 4 (r & 3) or u ^ 4 ((r / 2) & 1): so do the 4
+// rows x 4 units of a transposing read's half wave.
+// The longest query tiles start first.  Splits (few query tiles behind a long
+// prefix) write partials for attn_merge_kernel.
+// Why 128 queries: K and V pass LDS once per 128 queries (at 32 queries a wave
+// its operand reads, 256 cycles a stage, stay under the 1536 of its MFMAs).
+// Measured in place of 16-query launches of attn_kernel, 32 heads x 128, 1500
+// rows from position 0: 94 x 9.5 us (and 94 merges of 3.9 us) -> 56 us, 0.49
+// PFLOP/s of the MFMAs issued (P in two parts).  Bound by the softmax's vector
+// work beside the MFMAs.
+constexpr int kPromptQ = 128;
+constexpr int kPromptKeys = 64;
+
+template <int D>
+__global__ __launch_bounds__(256, 2) void attn_prompt_kernel(AttnArgs a)
+{
+    constexpr int RB = 2 * D, U = D / 8, TILE = kPromptKeys * RB;
+    constexpr int RPC = 1024 / RB;               // rows of a copy
+    constexpr int NC = kPromptKeys / RPC / 4;    // copies of a wave, of K and of V
+    __shared__ uint4 tiles[4 * TILE / 16];       // [buffer][K, V]
+    const char* const lds = (const char*)tiles;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)tiles;
+
+    const int h = blockIdx.x, qt = gridDim.y - 1 - blockIdx.y, s = blockIdx.z;
+    const int lane = threadIdx.x & 63, c = lane & 31, kg = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q0 = qt * kPromptQ, wq0 = q0 + 32 * wave;
+    const int Lt = a.n_prefix + min(a.nq, q0 + kPromptQ);  // keys some query of the tile sees
+    const int j0 = s * a.keys_per_split, j1 = min(Lt, j0 + a.keys_per_split);
+    if (j0 >= j1) return;
+    const int Lw = wq0 < a.nq ? a.n_prefix + min(a.nq, wq0 + 32) : 0;  // ... of the wave (none: it only copies)
+    const int qi = min(wq0 + c, a.nq - 1);  // rows past the last repeat it and are not stored
+    const int jq = a.n_prefix + qi;         // its last visible key
+
+    const size_t row_stride = (size_t)a.Hkv * D;
+    const size_t head = (size_t)(h / (a.H / a.Hkv)) * D;
+    const uint32_t rs2 = (uint32_t)row_stride * 2u;
+    uint32_t koff[NC], voff[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const int r = (wave + 4 * i) * RPC + lane / U, u = lane % U;
+        const int fk = D == 128 ? r & 15 : (r >> 1) & 7, fv = D == 128 ? (r & 3) << 2 : ((r >> 1) & 1) << 2;
+        koff[i] = (uint32_t)r * rs2 + (uint32_t)(u ^ fk) * 16u;
+        voff[i] = (uint32_t)r * rs2 + (uint32_t)(u ^ fv) * 16u;
+    }
+    // rows past the last key read 0
+    auto copy = [&](int j, int buf) {
+        const size_t at = (size_t)j * row_stride + head;
+        const uint32_t bytes = (uint32_t)(min(kPromptKeys, j1 - j) - 1) * rs2 + RB;
+        const rsrc_words kr = make_words(a.k + at, bytes), vr = make_words(a.v + at, bytes);
+        const uint32_t to = lds0 + (uint32_t)(buf * 2 * TILE + wave * 1024);
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            copy_lds(kr, to + 4096 * i, koff[i], 0);
+            copy_lds(vr, to + TILE + 4096 * i, voff[i], 0);
+        }
+    };
+    copy(j0, 0);
+
+    half8_t qb[D / 16];
+#pragma unroll
+    for (int st = 0; st < D / 16; ++st)
+        qb[st] = *(const half8_t*)(a.q + ((size_t)qi * a.H + h) * D + 16 * st + 8 * kg);
+    int ka[D / 16], va[D / 32];  // K row c, unit 2 st + kg; V row 4 kg + (lane / 4) % 4, this lane's 4 columns of tile dt
+#pragma unroll
+    for (int st = 0; st < D / 16; ++st) {
+        const int fk = D == 128 ? c & 15 : (c >> 1) & 7;
+        ka[st] = c * RB + (((2 * st + kg) ^ fk) << 4);
+    }
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt) {
+        const int r = (lane >> 2) & 3, fv = D == 128 ? r : r >> 1;
+        va[dt] = (4 * kg + r) * RB + ((4 * (dt ^ fv) + 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1)) << 4) + 8 * (lane & 1);
+    }
+
+    float m = -INFINITY, l = 0.0f;  // l: this lane's keys
+    float16_t o[D / 32];
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt) o[dt] = zero16();
+    for (int j = j0, buf = 0; j < j1; j += kPromptKeys, buf ^= 1) {
+        vm_wait<0>();  // this wave's copies of the stage
+        lds_barrier();
+        if (j + kPromptKeys < j1) copy(j + kPromptKeys, buf ^ 1);
+        if (j >= Lw) continue;  // uniform in the wave
+        const char* const kt = lds + buf * 2 * TILE;
+        const char* const vt = kt + TILE;
+        float16_t sc[2] = {zero16(), zero16()};
+#pragma unroll
+        for (int st = 0; st < D / 16; ++st)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) sc[t] = mfma32x32x16(*(const half8_t*)(kt + ka[st] + 32 * RB * t), qb[st], sc[t]);
+        // lane holds S^T[key 32 t + 8 (i / 4) + 4 kg + i % 4][query c]
+        if (j + kPromptKeys - 1 > a.n_prefix + wq0) {  // uniform: some key is hidden from some query
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (j + 32 * t + 8 * (i >> 2) + 4 * kg + (i & 3) > jq) sc[t][i] = -INFINITY;
+        }
+        float tmax = -INFINITY;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, sc[t][i]);
+        tmax = fmaxf(tmax, xor_lane<32>(tmax));
+        const float mnew = fmaxf(m, tmax * a.scale_log2);
+        const float muse = mnew == -INFINITY ? 0.0f : mnew;
+        if (__any(mnew > m)) {
+            const float alpha = exp2_fast(m - muse);
+            l *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < D / 32; ++dt) o[dt] = o[dt] * alpha;
+        }
+        m = mnew;
+        half8_t phi[4], plo[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float p = exp2_fast(__builtin_fmaf(sc[t >> 1][8 * (t & 1) + e], a.scale_log2, -muse));
+                l += p;
+                phi[t][e] = (_Float16)p;
+                plo[t][e] = (_Float16)(p - (float)phi[t][e]);
+            }
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int dt = 0; dt < D / 32; ++dt) {
+                short4_t v4[2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    v4[e] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (__attribute__((address_space(3))) short4_t*)(vt + va[dt] + (16 * t + 8 * e) * RB));
+                const half8_t v = __builtin_bit_cast(half8_t, __builtin_shufflevector(v4[0], v4[1], 0, 1, 2, 3, 4, 5, 6, 7));
+                o[dt] = mfma32x32x16(v, phi[t], o[dt]);
+                o[dt] = mfma32x32x16(v, plo[t], o[dt]);
+            }
+    }
+    l += xor_lane<32>(l);
+    if (wq0 + c >= a.nq) return;
+    // lane holds O^T[d = 32 dt + 8 (i / 4) + 4 kg + i % 4][query c]
+    float* const pp = a.part + (((size_t)h * a.splits + s) * a.nq + qi) * (D + 2);
+    _Float16* const hi = (_Float16*)a.out + ((size_t)qi * a.H + h) * D;
+    _Float16* const lo = hi + (size_t)a.nq * a.H * D;
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+            const int d = 32 * dt + 8 * i4 + 4 * kg;
+            if (a.splits == 1) {
+                half4_t vh, vl;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    _Float16 x, y;
+                    split_hl(o[dt][4 * i4 + i] / l, x, y);
+                    vh[i] = x;
+                    vl[i] = y;
+                }
+                *(half4_t*)(hi + d) = vh;
+                *(half4_t*)(lo + d) = vl;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; i += 2)
+                    *(float2*)(pp + d + i) = float2{o[dt][4 * i4 + i], o[dt][4 * i4 + i + 1]};
+            }
+        }
+    if (a.splits > 1 && kg == 0) *(float2*)(pp + D) = float2{m, l};
+}
+
+template <int D>
+void launch_merge(const AttnArgs& a, hipStream_t st)
+{
+    const dim3 mg(a.H, a.nq, a.nseq);
+    if (a.splits <= 16) hipLaunchKernelGGL((attn_merge_kernel<D, 16>), mg, dim3(D), 0, st, a);
+    else if (a.splits <= 32) hipLaunchKernelGGL((attn_merge_kernel<D, 32>), mg, dim3(D), 0, st, a);
+    else hipLaunchKernelGGL((attn_merge_kernel<D, kAttnMaxSplits>), mg, dim3(D), 0, st, a);
+}
+
 template <int D>
 void launch_attn(const AttnArgs& a, int T, hipStream_t st)
 {
@@ -308,12 +504,15 @@ void launch_attn(const AttnArgs& a, int T, hipStream_t st)
     case 2: hipLaunchKernelGGL((attn_kernel<D, 2>), grid, block, 0, st, a); break;
     default: hipLaunchKernelGGL((attn_kernel<D, 4>), grid, block, 0, st, a); break;
     }
-    if (a.splits > 1) {
-        const dim3 mg(a.H, a.nq, a.nseq);
-        if (a.splits <= 16) hipLaunchKernelGGL((attn_merge_kernel<D, 16>), mg, dim3(D), 0, st, a);
-        else if (a.splits <= 32) hipLaunchKernelGGL((attn_merge_kernel<D, 32>), mg, dim3(D), 0, st, a);
-        else hipLaunchKernelGGL((attn_merge_kernel<D, kAttnMaxSplits>), mg, dim3(D), 0, st, a);
-    }
+    if (a.splits > 1) launch_merge<D>(a, st);
+}
+
+template <int D>
+void launch_prompt(const AttnArgs& a, hipStream_t st)
+{
+    const dim3 grid(a.H, (a.nq + kPromptQ - 1) / kPromptQ, a.splits);
+    hipLaunchKernelGGL((attn_prompt_kernel<D>), grid, dim3(256), 0, st, a);
+    if (a.splits > 1) launch_merge<D>(a, st);
 }
 
 }  // namespace
@@ -369,6 +568,7 @@ ulspec_status attn_launch(ulspec_ctx* ctx, const AttnCall& c)
     a.n_prefix = (int)c.n_prefix;  // with dyn_prefix: the largest prefix the call may see
     a.nq = (int)c.nq;
     a.L = (int)(c.n_prefix + c.nq);
+    a.q_tile = 0;
     a.H = (int)c.H;
     a.Hkv = (int)c.Hkv;
     a.scale_log2 = c.scale * 1.4426950408889634f;
@@ -405,6 +605,64 @@ ulspec_status attn_launch(ulspec_ctx* ctx, const AttnCall& c)
     if (c.D == 128) launch_attn<128>(a, T, ctx->stream);
     else launch_attn<64>(a, T, ctx->stream);
     return check_launch(ctx, "verify_attention launch");
+}
+
+namespace {
+
+// Splits of a prompt of nq rows over L keys: about two workgroups per CU (what
+// LDS holds), at least two stages of keys each.
+void prompt_plan(int nq, int L, int H, int n_cu, int& splits, int& kps)
+{
+    const int tiles = (nq + kPromptQ - 1) / kPromptQ;
+    const int want = std::max(1, std::min((int)(2LL * n_cu / ((int64_t)tiles * H)), kAttnMaxSplits));
+    kps = std::max(2, ((L + want - 1) / want + kPromptKeys - 1) / kPromptKeys) * kPromptKeys;
+    splits = (L + kps - 1) / kps;
+}
+
+}  // namespace
+
+size_t attn_prompt_bytes(int rows, int max_ctx, int H, int D, int n_cu)
+{
+    size_t most = 0;
+    for (int q = std::min(rows, kPromptQ);; q = std::min(rows, q + kPromptQ)) {
+        const int tiles = (q + kPromptQ - 1) / kPromptQ;
+        const int64_t s = std::min<int64_t>({2LL * n_cu / ((int64_t)tiles * H), kAttnMaxSplits,
+                                             (max_ctx + 2 * kPromptKeys - 1) / (2 * kPromptKeys)});
+        if (s > 1) most = std::max(most, attn_workspace_bytes((int)s, H, q, D, 1));
+        if (q == rows) return most;
+    }
+}
+
+ulspec_status attn_prompt_launch(ulspec_ctx* ctx, const AttnCall& c)
+{
+    if (c.nq == 0 || (c.D != 64 && c.D != 128) || c.H == 0 || c.Hkv == 0 || c.H % c.Hkv || c.nseq != 1 || c.parent ||
+        !c.out_split || c.dyn_prefix || (uint64_t)c.n_prefix + c.nq > (uint64_t)INT32_MAX - kPromptKeys ||
+        (uint64_t)c.Hkv * c.D * 2 * kPromptKeys > (uint64_t)INT32_MAX)
+        return fail(ctx, ULSPEC_EINVAL, "prompt attention: %u rows at %u, H=%u Hkv=%u D=%u", c.nq, c.n_prefix, c.H, c.Hkv,
+                    c.D);
+    AttnArgs a{};
+    a.q = (const _Float16*)c.q;
+    a.k = (const _Float16*)c.k_cache;
+    a.v = (const _Float16*)c.v_cache;
+    a.out = c.out;
+    a.out_mode = 2;
+    a.nseq = 1;
+    a.n_prefix = (int)c.n_prefix;
+    a.nq = (int)c.nq;
+    a.L = (int)(c.n_prefix + c.nq);
+    a.q_tile = kPromptQ;
+    a.H = (int)c.H;
+    a.Hkv = (int)c.Hkv;
+    a.scale_log2 = c.scale * 1.4426950408889634f;
+    prompt_plan(a.nq, a.L, a.H, ctx->n_cu, a.splits, a.keys_per_split);
+    a.part = (float*)c.part;
+    const size_t need = attn_workspace_bytes(a.splits, a.H, a.nq, (int)c.D, 1);
+    if (need > c.part_bytes)
+        return fail(ctx, ULSPEC_EINVAL, "prompt attention: %d splits need %zu B of partials, the workspace holds %zu B",
+                    a.splits, need, c.part_bytes);
+    if (c.D == 128) launch_prompt<128>(a, ctx->stream);
+    else launch_prompt<64>(a, ctx->stream);
+    return check_launch(ctx, "prompt attention launch");
 }
 
 }  // namespace ulspec

@@ -58,20 +58,6 @@ constexpr int kUnitsPerChunk = kSuperBlock<TYPE> ? 32 : 16;
 // The hardware still overlaps them; s_waitcnt is placed at each first use.
 __device__ __forceinline__ void pin_loads() { asm volatile("" ::: "memory"); }
 
-// Workgroup barrier after this wave's LDS accesses have completed; no memory
-// fence, so vector loads in flight stay in flight across it.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// Wait until every vector-memory operation but the N youngest has completed;
-// no barrier.  After this wave's own buffer->LDS copies followed by N register
-// loads, the wave may read what it copied.
-template <int N>
-__device__ __forceinline__ void vm_wait()
-{
-    static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 #define ULSPEC_VM_CASE(n) \
     case n: vm_wait<n>(); break;
 #define ULSPEC_VM_CASE8(n) \

@@ -40,8 +40,6 @@
 
 using namespace ulspec;
 
-typedef float float16_t __attribute__((ext_vector_type(16)));
-
 namespace {
 
 constexpr int kTileWaves = 8;
@@ -232,16 +230,6 @@ __device__ __forceinline__ void tile_dequant(const TileRaw<TYPE>& w, const Nibbl
     }
 }
 
-__device__ __forceinline__ float16_t mfma32x32x16(half8_t a, half8_t b, float16_t c)
-{
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ float16_t zero16()
-{
-    return float16_t{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-}
-
 // f(integral_constant 0) .. f(integral_constant N - 1): a loop whose indexes are
 // constants before any optimisation, so register arrays stay in registers.
 template <class F, int... I>
@@ -261,24 +249,6 @@ __device__ __forceinline__ void pin(float16_t& v)
 {
     asm volatile("" : "+v"(v));
     __builtin_amdgcn_sched_barrier(0);
-}
-
-// 64 lanes' 16 bytes at their offsets (plus soff) -> LDS bytes at .. at + 1023.  Written
-// out because behind the builtin every LDS read waits for all copies in
-// flight (the reads and the copies could alias); here the one wait is the
-// loop's, before its barrier.  (m0 needs one wait state before its use.)
-typedef uint32_t rsrc_words __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ rsrc_words make_words(const void* base, uint32_t bytes)
-{
-    const uint64_t p = (uint64_t)base;
-    return rsrc_words{(uint32_t)p, (uint32_t)(p >> 32) & 0xffffu, bytes, 0x00020000u};
-}
-
-__device__ __forceinline__ void copy_lds(rsrc_words r, uint32_t at, uint32_t off, uint32_t soff)
-{
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :: "s"(at), "v"(off), "s"(r), "s"(soff) : "memory", "m0");
 }
 
 constexpr size_t tile_lds_bytes(int rows) { return (size_t)2 * rows * 512 + (size_t)2 * rows * 32; }
@@ -622,6 +592,11 @@ bool gemm_tile_wins(const Weight& w, uint32_t M)
 size_t gemm_tile_workspace_bytes(const Weight& w, int n_cu)
 {
     return tile_sum_bytes(w, kTileRowsH16) + (size_t)std::max(1, n_cu) * 128 * kTileCols * sizeof(float);
+}
+
+size_t gemm_tile_split_bytes(uint32_t M, uint32_t K, int n_cu)
+{
+    return align256((size_t)2 * M * (K / 8)) + (size_t)std::max(1, n_cu) * 64 * kTileCols * sizeof(float);
 }
 
 ulspec_status gemm_tile(ulspec_ctx* ctx, const Weight& w, const GemmFuse& f, const uint16_t* x, uint32_t M, bool hl,

@@ -9,6 +9,7 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef float float16_t __attribute__((ext_vector_type(16)));
 
 namespace ulspec {
 
@@ -96,6 +97,51 @@ __device__ __forceinline__ float4_t mfma16x16x32(half8_t a, half8_t b, float4_t 
 __device__ __forceinline__ float4_t mfma16x16x16(half4_t a, half4_t b, float4_t c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
+}
+
+// 32x32x16 fp16 MFMA: lane l supplies row (A) or column (B) l & 31 and 8 K
+// values of half kg = l >> 5, and holds C rows 8 (i / 4) + 4 kg + i % 4 of
+// column l & 31.
+__device__ __forceinline__ float16_t mfma32x32x16(half8_t a, half8_t b, float16_t c)
+{
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ float16_t zero16()
+{
+    return float16_t{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+}
+
+// Workgroup barrier after this wave's LDS accesses have completed; no memory
+// fence, so vector loads in flight stay in flight across it.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Wait until every vector-memory operation but the N youngest has completed;
+// no barrier.  After this wave's own buffer->LDS copies followed by N register
+// loads, the wave may read what it copied.
+template <int N>
+__device__ __forceinline__ void vm_wait()
+{
+    static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// 64 lanes' 16 bytes at their offsets (plus soff) -> LDS bytes at .. at + 1023.  Written
+// out because behind the builtin every LDS read waits for all copies in
+// flight (the reads and the copies could alias); here the one wait is the
+// loop's, before its barrier.  (m0 needs one wait state before its use.)
+typedef uint32_t rsrc_words __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ rsrc_words make_words(const void* base, uint32_t bytes)
+{
+    const uint64_t p = (uint64_t)base;
+    return rsrc_words{(uint32_t)p, (uint32_t)(p >> 32) & 0xffffu, bytes, 0x00020000u};
+}
+
+__device__ __forceinline__ void copy_lds(rsrc_words r, uint32_t at, uint32_t off, uint32_t soff)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :: "s"(at), "v"(off), "s"(r), "s"(soff) : "memory", "m0");
 }
 
 }  // namespace ulspec

@@ -43,25 +43,29 @@ struct ulspec_model {
     float2* rope = nullptr;    // [max_ctx][head_dim / 2] (cos, sin)
 
     // activations, up to rows_cap rows per forward (kRows per sequence;
-    // n_seq sequence slots, each with its own K / V cache).  GEMM inputs are
+    // n_seq sequence slots, each with its own K / V cache), or rows_prompt rows
+    // of one sequence's prompt (what a row needs through the layers; R in the
+    // sizes below is the larger of the two).  GEMM inputs are
     // fp32 activations held as split fp16 pairs [2 rows][width] (high parts,
     // then low parts): the attention output and SiLU(gate) * up.
     static constexpr uint32_t kRows = 16;
     static constexpr uint32_t kBatchRows = 48;  // rows of a batched forward (8 sequences x 6)
     uint32_t rows_max = 0;     // rows of one sequence per forward
     uint32_t rows_cap = 0;     // rows of all sequences of one forward
+    static constexpr uint32_t kPromptRows = 2048;
+    uint32_t rows_prompt = 0;  // rows of one prompt forward
     uint32_t n_seq = 1;
-    float* h = nullptr;        // [kRows][dim] residual stream (fp32)
-    float* pss = nullptr;      // [kRows][pss_stride] RMSNorm partial sums of h^2
+    float* h = nullptr;        // [R][dim] residual stream (fp32)
+    float* pss = nullptr;      // [R][pss_stride] RMSNorm partial sums of h^2
     uint32_t pss_stride = 0;
     float* logits = nullptr;   // [kRows][vocab]
-    _Float16* q16 = nullptr;   // [kRows][H D] (attention queries, fp16)
-    _Float16* att = nullptr;   // split [2 kRows][H D]
-    _Float16* act = nullptr;   // split [2 kRows][F]
-    _Float16* xn = nullptr;    // split [2 kRows][dim]: h times the next RMSNorm's weights (the next GEMM's X)
-    float* part = nullptr;     // split-K slice partials
+    _Float16* q16 = nullptr;   // [R][H D] (attention queries, fp16)
+    _Float16* att = nullptr;   // split [2 R][H D]
+    _Float16* act = nullptr;   // split [2 R][F]
+    _Float16* xn = nullptr;    // split [2 R][dim]: h times the next RMSNorm's weights (the next GEMM's X)
+    float* part = nullptr;     // split-K slice partials, row sums of the many-row GEMM
     size_t part_bytes = 0;
-    int32_t* tok = nullptr;    // [kRows]
+    int32_t* tok = nullptr;    // [R]
     int32_t* pos = nullptr;    // [1]
     int32_t* lin_pos = nullptr;  // [1] the position of ulspec_model_linear calls
     int64_t lin_pos_set = -1;    // the value last written there (-1: none)
@@ -101,8 +105,16 @@ struct ulspec_model {
     ulspec_status forward(const int32_t* tok_dev, uint32_t M, const int32_t* pos_dev, int32_t pos_add,
                           float* logits_dev, uint32_t n_logits, const int32_t* parent = nullptr, uint32_t nseq = 1,
                           uint32_t seq0 = 0);
-    // Host tokens on sequence slot seq (chunks of rows_max rows), logits of the
-    // last n_logits rows to host memory.  Synchronous.
+    // The same for M <= rows_prompt rows of one sequence from position pos (as
+    // in m->pos), n_logits <= rows_max.
+    ulspec_status forward_prompt(const int32_t* tok_dev, uint32_t M, uint32_t pos, float* logits_dev, uint32_t n_logits,
+                                 uint32_t seq);
+    // The layers and the head behind both; prompt: the rows attend by
+    // attn_prompt_launch from position prompt_pos.
+    ulspec_status run_layers(const int32_t* tok_dev, const Rows& rows, const int32_t* parent, float* logits_dev,
+                             uint32_t n_logits, bool prompt, uint32_t prompt_pos);
+    // Host tokens on sequence slot seq (more than rows_max rows: in prompt
+    // chunks), logits of the last n_logits rows to host memory.  Synchronous.
     ulspec_status forward_host(const int32_t* tokens, uint32_t M, uint32_t pos, float* logits, uint32_t n_logits,
                                uint32_t seq);
 };

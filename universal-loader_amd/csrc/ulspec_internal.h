@@ -131,8 +131,8 @@ ulspec_status rows_to_f16(ulspec_ctx* ctx, uint32_t type, const void* raw, uint3
                           _Float16* out, uint32_t out_row0, uint32_t out_row_step);
 // The dequant-GEMM with a fused row scale / epilogue over split X (the model
 // forward; the low part of row m at row lo_rows + m): the whole-X kernels for
-// M <= 8 rows that fit in LDS, else the split-K kernel and the reducing
-// epilogue.
+// M <= 8 rows that fit in LDS, the split-K kernel and the reducing epilogue up
+// to kGemmRowsSplit rows, else the many-row kernel.
 ulspec_status gemm_fused(ulspec_ctx* ctx, const Weight& w, const GemmFuse& f, const uint16_t* x, uint32_t M,
                          uint32_t lo_rows, float* y);
 // The many-row dequant-GEMM (gemm_tile.hip): fp16 X (hl false) or split X (the
@@ -142,6 +142,8 @@ constexpr uint32_t kTileRowsH16 = 4096;
 bool gemm_tile_wins(const Weight& w, uint32_t M);
 ulspec_status gemm_tile_init(ulspec_ctx* ctx);
 size_t gemm_tile_workspace_bytes(const Weight& w, int n_cu);
+// The same for split X of M rows and K elements each (any weight type).
+size_t gemm_tile_split_bytes(uint32_t M, uint32_t K, int n_cu);
 ulspec_status gemm_tile(ulspec_ctx* ctx, const Weight& w, const GemmFuse& f, const uint16_t* x, uint32_t M, bool hl,
                         uint32_t lo_rows, float* y, void* ws, size_t ws_bytes);
 size_t gemm_workspace_bytes(const Weight& w);
@@ -171,6 +173,11 @@ struct AttnCall {
     size_t kv_seq = 0;
 };
 ulspec_status attn_launch(ulspec_ctx* ctx, const AttnCall& c);
+// A prompt's rows on one sequence: causal, n_prefix cached keys (host value)
+// before nq rows (any number), split fp16 output; partials of at most
+// attn_prompt_bytes for calls of up to `rows` rows within max_ctx.
+ulspec_status attn_prompt_launch(ulspec_ctx* ctx, const AttnCall& c);
+size_t attn_prompt_bytes(int rows, int max_ctx, int H, int D, int n_cu);
 void attn_plan(int L, int H, int n_cu, int& splits, int& kps);
 size_t attn_workspace_bytes(int splits, int H, int nq, int D, int nseq = 1);
 size_t accept_workspace_bytes(uint32_t B, uint32_t k);
