@@ -18,6 +18,8 @@ CASES = [
     (8, 4096, 2048, (129,)),
     (1, 257, 416, (17, 64, 129)),
     (1, 2048, 2048, (500,)),
+    (2, 4096, 1536, (2080,)),         # 272 blocks: a whole round, then 16 sliced ones
+    (12, 17000, 1024, (513, 640)),    # a last round of 79 blocks
 ]
 
 

@@ -24,10 +24,6 @@ struct GemmArgs {
     GemmFuse f;      // row scale and epilogue
 };
 
-// The sum of a.ks_count slices of part [ks][M][N] (host; asynchronous), row
-// scale and a.f's epilogue into a.out.
-void gemm_reduce_launch(ulspec_ctx* ctx, const GemmArgs& a, const float* part);
-
 namespace {
 
 constexpr int kQ40Chunk = 1152;

@@ -31,7 +31,7 @@
 // reads and dequantizes the whole weight once per 64 rows), at 2048 x 11008 x
 // 4096: Q4_K 869 -> 202 us (0.92 PFLOP/s), Q4_0 240, Q8_0 266 (a block's scale
 // per 32 K: twice the accumulator updates of the super-block types), Q6_K 217,
-// F16 214 us; 333 x 4096 x 4096 Q8_0 79.9 -> 32.8 us.  Bound by the vector unit
+// F16 214 us; 333 x 4096 x 4096 Q8_0 79.9 -> 32.3 us.  Bound by the vector unit
 // beside the matrix cores: dequantization, and the scaling of every product.
 #include "gemm_dev.h"
 
@@ -51,10 +51,25 @@ struct TileArgs {
     const uint4* xsum;  // Q4_K: sub-block sums of X (tile_sums_kernel), [K / 256][xsum_rows][2]
     int xsum_rows;
     int n_stages;       // ceil(K / 256)
-    int st_q, st_r;     // n_stages = st_q * ks_count + st_r
     int tm, tn;         // row and column blocks
-    int direct;         // epilogue here; else fp32 slice partials to a.out[ks][M][N]
+    // Blocks 0 .. n_full - 1 take a workgroup each, the n_part others a.ks_count
+    // workgroups: slices of st_q or st_q + 1 stages (n_stages = st_q ks_count +
+    // st_r), left as fp32 parts for tile_fixup_kernel.
+    int n_full, n_part;
+    int st_q, st_r;
+    float* part;        // [n_part][ks_count][rows of a block][kTileCols]
 };
+
+// Row and column block i: 8 row blocks before the next column block, so the ~32
+// resident workgroups of an XCD share 8 X blocks and a few weight blocks in its L2.
+__device__ __forceinline__ void block_at(const TileArgs& ta, int i, int& mb, int& nb)
+{
+    constexpr int GM = 8;
+    const int grp = i / (GM * ta.tn), first = grp * GM, in = i - grp * GM * ta.tn;
+    const int gm = min(GM, ta.tm - first);
+    mb = first + in % gm;
+    nb = in / gm;
+}
 
 // One stage of a wave's weights as loaded: the chunk pieces of lane groups kg
 // and kg + 2.
@@ -271,17 +286,15 @@ __global__ __launch_bounds__(kTileWaves * 64, 2) void gemm_tile_kernel(TileArgs 
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)tile_lds;
     const GemmArgs& a = ta.a;
 
-    // Blocks of one XCD (blockIdx.x % 8) are consecutive in an order that runs
-    // through 8 row blocks before the next column block: the ~32 resident
-    // blocks of an XCD share 8 X blocks and a few weight blocks in its L2.
-    const int nblk = ta.tm * ta.tn, total = nblk * a.ks_count;
-    const int id = (int)(blockIdx.x % kTileXcds) * ((total + kTileXcds - 1) / kTileXcds) + (int)(blockIdx.x / kTileXcds);
-    if (id >= total) return;
-    const int ks = id / nblk, rest = id - ks * nblk;
-    constexpr int GM = 8;
-    const int grp = rest / (GM * ta.tn), first = grp * GM, in = rest - grp * GM * ta.tn;
-    const int gm = min(GM, ta.tm - first);
-    const int mb = first + in % gm, nb = in / gm;
+    // Workgroups of one XCD (blockIdx.x % 8) are consecutive blocks, or slices of
+    // blocks, of the order of block_at.
+    const bool sliced = (int)blockIdx.x >= ta.n_full;
+    const int count = sliced ? ta.n_part * a.ks_count : ta.n_full, bid = (int)blockIdx.x - (sliced ? ta.n_full : 0);
+    const int per = count / kTileXcds, extra = count % kTileXcds, xcd = bid % kTileXcds;
+    const int id = xcd * per + min(xcd, extra) + bid / kTileXcds;
+    const int ks = sliced ? id / ta.n_part : 0, u = id - ks * ta.n_part;
+    int mb, nb;
+    block_at(ta, sliced ? ta.n_full + u : id, mb, nb);
 
     const int lane = threadIdx.x & 63, kg = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -343,7 +356,8 @@ __global__ __launch_bounds__(kTileWaves * 64, 2) void gemm_tile_kernel(TileArgs 
         return *(const half8_t*)(lds + buf * BUF + o + mt * 4096);
     };
 
-    int lo = ks * ta.st_q + min(ks, ta.st_r), hi = lo + ta.st_q + (ks < ta.st_r ? 1 : 0);
+    const int lo = sliced ? ks * ta.st_q + min(ks, ta.st_r) : 0;
+    const int hi = sliced ? lo + ta.st_q + (ks < ta.st_r ? 1 : 0) : ta.n_stages;
     float16_t acc[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[mt] = zero16();
@@ -435,15 +449,25 @@ __global__ __launch_bounds__(kTileWaves * 64, 2) void gemm_tile_kernel(TileArgs 
     // accumulator i of tile mt: row 32 mt + 8 (i / 4) + 4 kg + i % 4
     constexpr int MO = HL ? MT / 2 : MT;
     if constexpr (HL) unrolled<MO>([&](auto mt) { acc[mt] = acc[mt] + acc[MO + mt] * kLoUnscale; });
-    if (!HL || !ta.direct) {  // fp16 X has no epilogue of its own
-        float* out = a.out + (size_t)ks * a.M * a.N;
+    if (sliced) {
+        // (Parts as [slice][M][N] instead: rows a power of two apart when N is; 4096 x
+        // 4096 Q4_K at 128 rows 23.6 -> 28.2 us, level elsewhere.)
+        float* out = ta.part + ((size_t)u * a.ks_count + ks) * RB * kTileCols + 32 * wave + (lane & 31);
         unrolled<MO>([&](auto mt) {
             unrolled<16>([&](auto i) {
-                const int m = m0 + 32 * mt + 8 * (i >> 2) + 4 * kg + (i & 3);
-                if (m < a.M && n < a.N) out[(size_t)m * a.N + n] = acc[mt][(int)i];
+                const int r = 32 * mt + 8 * (i >> 2) + 4 * kg + (i & 3);
+                if (m0 + r < a.M) out[r * kTileCols] = acc[mt][(int)i];
             });
         });
         return;
+    }
+    if constexpr (!HL) {  // fp16 X has no epilogue
+        unrolled<MO>([&](auto mt) {
+            unrolled<16>([&](auto i) {
+                const int m = m0 + 32 * mt + 8 * (i >> 2) + 4 * kg + (i & 3);
+                if (m < a.M && n < a.N) a.out[(size_t)m * a.N + n] = acc[mt][(int)i];
+            });
+        });
     }
     if constexpr (HL) {
         float* rs = (float*)lds;
@@ -468,6 +492,52 @@ __global__ __launch_bounds__(kTileWaves * 64, 2) void gemm_tile_kernel(TileArgs 
                 epilogue(a, s, m0 + r0 + i, n, n >> 4, lane, pre[i], pos0);
             });
         });
+    }
+}
+
+// The sliced blocks: their slices summed in K order, then the row scale and
+// epilogue.  Grid (n_part, rows of a block / RPT), a thread per column; SU >=
+// ks_count reads a row are issued before the first add.
+template <int SU, int RPT>
+__global__ __launch_bounds__(kTileCols) void tile_fixup_kernel(TileArgs ta, int rb)
+{
+    static_assert(RPT <= kTileCols / 64, "one wave per row scale");
+    __shared__ float rs[RPT];
+    const GemmArgs& a = ta.a;
+    // the parts are read whatever M and N are (they hold whole blocks), ahead of the block's place
+    const int r0 = (int)blockIdx.y * RPT;
+    const size_t slice = (size_t)rb * kTileCols;
+    const float* p = ta.part + (size_t)blockIdx.x * a.ks_count * slice + (size_t)r0 * kTileCols + threadIdx.x;
+    float v[RPT][SU];
+#pragma unroll
+    for (int j = 0; j < RPT; ++j)
+#pragma unroll
+        for (int k = 0; k < SU; ++k) v[j][k] = k < a.ks_count ? p[k * slice + j * kTileCols] : 0.0f;
+    int mb, nb;
+    block_at(ta, ta.n_full + (int)blockIdx.x, mb, nb);
+    const int m0 = mb * rb + r0;
+    if (m0 >= a.M) return;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = nb * kTileCols + (int)threadIdx.x;
+    const EpiPos pos0 = epi_pos0(a);
+    float2 pre[RPT];
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) pre[j] = epi_load(a, m0 + j, n, pos0);
+    if (a.f.rs_pss) {
+        if (wave < RPT && m0 + wave < a.M) {  // wave-uniform
+            const float r = rs_reduce(a, rs_load(a, m0 + wave));
+            if (lane == 0) rs[wave] = r;
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+        float s = v[j][0];
+#pragma unroll
+        for (int k = 1; k < SU; ++k) s = k < a.ks_count ? s + v[j][k] : s;
+        if (a.f.rs_pss) s *= rs[j];
+        if (m0 + j < a.M) epilogue(a, s, m0 + j, n, n >> 4, lane, pre[j], pos0);
     }
 }
 
@@ -500,8 +570,7 @@ __global__ __launch_bounds__(256) void tile_sums_kernel(const uint4* __restrict_
 template <int TYPE, int MT, bool HL>
 void tile_launch(const TileArgs& ta, hipStream_t st)
 {
-    const int total = ta.tm * ta.tn * ta.a.ks_count;
-    const int grid = (total + kTileXcds - 1) / kTileXcds * kTileXcds;
+    const int grid = ta.n_full + ta.n_part * ta.a.ks_count;
     hipLaunchKernelGGL((gemm_tile_kernel<TYPE, MT, HL>), dim3(grid), dim3(kTileWaves * 64), tile_lds_bytes(32 * MT), st,
                        ta);
 }
@@ -555,12 +624,42 @@ namespace {
 // 32-row operand tiles of a workgroup for M rows of fp16 X.
 int tile_mt(uint32_t M) { return M <= 32 ? 1 : M <= 64 ? 2 : 4; }
 
-// K slices: as many as fill the CUs once (a workgroup holds a CU's LDS), at
-// least two stages each; one for the blocks that already do.
-int tile_ksplit(const Weight& w, int blocks, int n_cu)
+// Slices of the rem blocks that do not fill a round of the CUs (a workgroup holds
+// a CU's LDS): those that minimise the rounds' length in stages of about 4 us, a
+// workgroup's start about one, plus the fix-up (its launch about three, and each
+// part's way through memory: rb rows of 1 KB twice, at about 20 MB a stage).  1:
+// no slices.  Slicing the last round only, against every block in n_cu / blocks
+// slices or none: split X of 1500 rows through the 7B layer (1152, 384, 2064 and
+// 384 blocks) 7.6 -> 7.1 ms per 4 layers, 12288 x 4096 Q4_K at 1500 rows 195 -> 177
+// us, 4096 x 4096 Q4_K at 128 27.3 -> 23.6, 6000 x 1024 F16 at 300 23.9 -> 16.9.
+// (The last round's stages dealt out evenly, as a loop over parts of two blocks:
+// 2048 x 11008 x 4096 Q4_K 202 -> 236 us, its parts being 56 MB.)
+constexpr float kTileStart = 1.0f, kTileFixup = 3.0f;
+constexpr int kTileMaxSlices = 32;
+int tile_slices(int rem, int stages, int rb, int n_cu)
 {
-    const int stages = (int)((w.k + 255) / 256);
-    return std::max(1, std::min(n_cu / std::max(1, blocks), stages / 2));
+    int best = 1;
+    float best_cost = (float)stages + kTileStart;
+    for (int ks = 2; ks <= std::min(stages / 2, kTileMaxSlices) && rem * ks <= 4 * n_cu; ++ks) {
+        const int rounds = (rem * ks + n_cu - 1) / n_cu;
+        const float cost = (float)rounds * ((float)((stages + ks - 1) / ks) + kTileStart) + kTileFixup +
+                           (float)rem * (float)ks * (float)rb * 1e-4f;
+        if (cost < best_cost) {
+            best = ks;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+template <int SU>
+void fixup_launch(const TileArgs& ta, int rb, int n_cu, hipStream_t st)
+{
+    const int rows = std::min(rb, ta.a.M), four = (rows + 3) / 4;
+    if (ta.n_part * four >= 2 * n_cu)
+        hipLaunchKernelGGL((tile_fixup_kernel<SU, 4>), dim3(ta.n_part, four), dim3(kTileCols), 0, st, ta, rb);
+    else
+        hipLaunchKernelGGL((tile_fixup_kernel<SU, 1>), dim3(ta.n_part, rows), dim3(kTileCols), 0, st, ta, rb);
 }
 
 size_t align256(size_t v) { return (v + 255) / 256 * 256; }
@@ -587,8 +686,8 @@ bool gemm_tile_wins(const Weight& w, uint32_t M)
     return M > 128 || (M > 64 && w.n > 2048) || (M > 16 && w.n > 8192);
 }
 
-// Workspace of the tile GEMM: the slice partials are at most one per CU (a
-// split fills the CUs at most once), the sums those of kTileRowsH16 rows.
+// Workspace of the tile GEMM: parts for one round of slices (gemm_tile takes
+// fewer where more would not fit), the sums those of kTileRowsH16 rows.
 size_t gemm_tile_workspace_bytes(const Weight& w, int n_cu)
 {
     return tile_sum_bytes(w, kTileRowsH16) + (size_t)std::max(1, n_cu) * 128 * kTileCols * sizeof(float);
@@ -626,16 +725,18 @@ ulspec_status gemm_tile(ulspec_ctx* ctx, const Weight& w, const GemmFuse& f, con
     ta.n_stages = (int)((w.k + 255) / 256);
     const size_t sums = tile_sum_bytes(w, xrows);
     if (sums > ws_bytes) return fail(ctx, ULSPEC_EINVAL, "tile gemm: %zu bytes of row sums, %zu available", sums, ws_bytes);
-    int ks = tile_ksplit(w, ta.tm * ta.tn, ctx->n_cu);
-    while (ks > 1 && sums + (size_t)ks * M * w.n * sizeof(float) > ws_bytes) --ks;
+    const int n_cu = std::max(1, ctx->n_cu), blocks = ta.tm * ta.tn, rem = blocks % n_cu;
+    int ks = rem ? tile_slices(rem, ta.n_stages, rb, n_cu) : 1;
+    while (ks > 1 && sums + (size_t)rem * ks * rb * kTileCols * sizeof(float) > ws_bytes) --ks;
+    ta.n_part = ks > 1 ? rem : 0;
+    ta.n_full = blocks - ta.n_part;
     a.ks_count = ks;
     ta.st_q = ta.n_stages / ks;
     ta.st_r = ta.n_stages % ks;
-    ta.direct = ks == 1;
     ta.xsum = (const uint4*)ws;
     ta.xsum_rows = (int)xrows;
-    float* part = (float*)((char*)ws + sums);
-    a.out = ks == 1 ? y : part;
+    ta.part = (float*)((char*)ws + sums);
+    a.out = y;
     if (w.type == ULSPEC_GGML_Q4_K)
         hipLaunchKernelGGL(tile_sums_kernel, dim3((w.k / 8 + 255) / 256, xrows), dim3(256), 0, ctx->stream,
                            (const uint4*)x, xrows, w.k, (half2_t*)ws);
@@ -645,8 +746,11 @@ ulspec_status gemm_tile(ulspec_ctx* ctx, const Weight& w, const GemmFuse& f, con
     else if (w.type == ULSPEC_GGML_Q8_0) tile_launch_t<ULSPEC_GGML_Q8_0>(ta, mt, ctx->stream);
     else tile_launch_t<ULSPEC_GGML_F16>(ta, mt, ctx->stream);
     if (ks > 1) {
-        a.out = y;
-        gemm_reduce_launch(ctx, a, part);
+        if (ks <= 2) fixup_launch<2>(ta, rb, n_cu, ctx->stream);
+        else if (ks <= 4) fixup_launch<4>(ta, rb, n_cu, ctx->stream);
+        else if (ks <= 8) fixup_launch<8>(ta, rb, n_cu, ctx->stream);
+        else if (ks <= 16) fixup_launch<16>(ta, rb, n_cu, ctx->stream);
+        else fixup_launch<kTileMaxSlices>(ta, rb, n_cu, ctx->stream);
     }
     return ULSPEC_OK;
 }
