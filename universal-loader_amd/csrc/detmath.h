@@ -10,19 +10,15 @@
 
 namespace ulspec {
 
-// exp(x): Cody & Waite reduction x = n ln2 + r (ln2 split in a 16-bit head
-// and a tail), degree-7 Taylor polynomial of e^r (error < r^8 / 8! < 2e-9
-// relative on |r| <= ln2/2), 2^n applied as two normal factors.  x < -87
-// gives 0 (every nonzero result is normal), x > 88.72 gives inf.
-__host__ __device__ inline float det_expf(float x)
+// e^r of the Cody & Waite reduction x = n ln2 + r (ln2 split in a 16-bit head
+// and a tail): degree-7 Taylor polynomial (error < r^8 / 8! < 2e-9 relative on
+// |r| <= ln2/2).
+__host__ __device__ inline float exp_poly(float x, float& n)
 {
-    if (!(x == x)) return x;
-    if (x < -87.0f) return 0.0f;
-    if (x > 88.72f) return __builtin_inff();
     const float log2e = 1.44269504088896341f;
     const float shifter = 12582912.0f;  // 1.5 * 2^23: round to nearest even
     const float t = __builtin_fmaf(x, log2e, shifter);
-    const float n = t - shifter;
+    n = t - shifter;
     const float ln2_hi = 0.693145751953125f;
     const float ln2_lo = 1.428606820309417232e-06f;
     float r = __builtin_fmaf(-n, ln2_hi, x);
@@ -34,7 +30,18 @@ __host__ __device__ inline float det_expf(float x)
     p = __builtin_fmaf(p, r, 1.66666666666666667e-01f);
     p = __builtin_fmaf(p, r, 0.5f);
     p = __builtin_fmaf(p, r, 1.0f);
-    p = __builtin_fmaf(p, r, 1.0f);
+    return __builtin_fmaf(p, r, 1.0f);
+}
+
+// exp(x): e^r with 2^n applied as two normal factors.  x < -87 gives 0 (every
+// nonzero result is normal), x > 88.72 gives inf.
+__host__ __device__ inline float det_expf(float x)
+{
+    if (!(x == x)) return x;
+    if (x < -87.0f) return 0.0f;
+    if (x > 88.72f) return __builtin_inff();
+    float n;
+    const float p = exp_poly(x, n);
     const int32_t ni = (int32_t)n;
     const int32_t n1 = ni / 2, n2 = ni - n1;
     const float s1 = __builtin_bit_cast(float, (uint32_t)(n1 + 127) << 23);
