@@ -21,8 +21,8 @@
 //   down  epilogue h += Y (+ sums of h^2)
 // and the LM head with the final RMSNorm in its prologue.  Rows up to 8 whose
 // split X fits in LDS run the whole-X kernels with both steps fused; others
-// (the 7B FFN width, trees and prefill chunks past 8 rows) the split-K kernel,
-// a norm kernel before it and the epilogue in its slice reduction.
+// (the 7B FFN width, trees and prompts past 8 rows) the split-K kernel with the
+// epilogue in its slice reduction, and past 48 rows (prompts) the many-row kernel.
 #include "model.h"
 
 #include <algorithm>
